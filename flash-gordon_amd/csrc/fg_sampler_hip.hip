@@ -1114,11 +1114,14 @@ fg_status fg_sampler_hip_create(fg_sampler_hip** out, uint32_t vocab, uint32_t m
   }
   if (e == hipSuccess) e = hipMalloc(&s->ws.params, sizeof(RowParams) * max_rows);
   if (e == hipSuccess) e = hipMalloc(&s->ws.cand, sizeof(uint64_t) * slots * fg::kMaxK);
-  // Hand-off slots start cleared (no word carries an epoch yet).
+  // Hand-off slots start cleared: no word carries an epoch yet.  (A block that
+  // an earlier sampler freed holds words of its first epochs, which are this
+  // one's too.)
   if (e == hipSuccess) e = hipMemset(s->ws.cand, 0, sizeof(uint64_t) * slots * fg::kMaxK);
   if (e == hipSuccess) e = hipMalloc(&s->ws.greedy, sizeof(uint64_t) * slots);
   if (e == hipSuccess) e = hipMemset(s->ws.greedy, 0, sizeof(uint64_t) * slots);
   if (e == hipSuccess) e = hipMalloc(&s->ws.spec, sizeof(uint64_t) * slots);
+  if (e == hipSuccess) e = hipMemset(s->ws.spec, 0, sizeof(uint64_t) * slots);
   if (e == hipSuccess) e = hipMalloc(&s->ws.lse, sizeof(double) * slots * 2);
   // (A workgroup slot each: wave slots / kWaves.)
   if (e == hipSuccess)
