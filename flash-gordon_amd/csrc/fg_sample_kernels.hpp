@@ -655,11 +655,11 @@ struct Features {
   static constexpr bool kLse = kLse_;      // log-probs requested
   static constexpr bool kNuc = kNuc_;      // some row is a whole-row nucleus (top_k 0)
   static constexpr bool kSpec = kSpec_;    // some top list is longer than kSpecMinK
-  // A finisher launch of more than 8 chunks a row with top lists (and neither
-  // log-probs nor whole-row nucleus rows): its rows' lists are selected from
-  // (many_select), the other hand-offs are compiled out.
+  // A launch of more than 8 chunks a row with top lists (and neither log-probs
+  // nor whole-row nucleus rows): its rows' lists are selected from
+  // (many_select), the other hand-offs of top lists are compiled out.
   static constexpr bool kMany = kMany_;
-  static_assert(!kMany || (kTop && !kLse && !kNuc), "a finisher launch");
+  static_assert(!kMany || (kTop && !kLse && !kNuc), "every row's list ranked in its workgroup");
   // Quads per lane per streaming step: 2 (512 elements) for launches
   // without speculation or whole-row nucleus rows, 4 otherwise (measured:
   // config 2 21.9 -> 21.1 us at 512, config 4 greedy 22.4 -> 21.8; top-k 64
@@ -1009,7 +1009,7 @@ __device__ inline uint64_t rescan_slice(const SampleArgs& a, const RowParams& p,
 // Every element a speculating wave skipped has a key below its key KS, so it
 // cannot enter the row's top-kk when KS is at most the key of the list's
 // kk-th entry; each wave of the row for which that fails is read again.
-// in_lds: ks_lds holds the keys (a row of one workgroup, a finisher of many
+// in_lds: ks_lds holds the keys (a row of one workgroup, the last of many
 // chunks); else they are read from the workspace.
 // The keys of waves 0..63 come in as ks0 (lane i: wave i), loaded early.
 __device__ __forceinline__ uint32_t spec_key(const SampleArgs& a, uint32_t row, uint32_t i,
@@ -1184,26 +1184,27 @@ __device__ __forceinline__ void rank_place_lists(const uint64_t* lists32, const 
 
 // ---- selecting from many lists ------------------------------------------------
 //
-// A finisher of more than 8 chunks (few rows: 1 row has 64) does not merge
-// its lists: all four waves read them into LDS, a bound from the lists' first
-// entries leaves little more than the kk best, and those are ranked among
-// themselves.  What bounds it is latency: the last arriver's rounds of eight
-// lists (one wave, a memory round trip each) took about 11 of the 23.5 us of
-// one row of 248,320 at top-k 20.  Measured, with the tagged words in place of
-// the arrival count: that row 23.5 -> 12.1 us; 8 rows, controls and history
-// increment included, 34.6 -> 21.8; 37 rows of 50,257, greedy and top-k 1-64
-// mixed, 17.9 -> 15.3 (with 16-byte loads for its unaligned rows).  Up to 8
-// lists the rank merge stays: it needs no bound.
+// The last workgroup of a row of more than 8 chunks (few rows: 1 row has 64)
+// does not merge the lists: all four waves read them into LDS, a bound from the
+// lists' first entries leaves little more than the kk best, and those are
+// ranked among themselves.  What bounds it is latency: rounds of eight lists
+// (one wave, a memory round trip each) took about 11 of the 23.5 us of one row
+// of 248,320 at top-k 20.  Measured, with the arrival count: that row 23.5 -> 12.7 us;
+// 8 rows, controls and history increment included, 34.6 -> 22.0; 37 rows of
+// 50,257, greedy and top-k 1-64 mixed, 17.9 -> 15.6 (with 16-byte loads for its
+// unaligned rows).  Tagged words in place of the count, whose reader waits for
+// the row's other chunks within a limit, gave 12.3, 22.1 and 15.6: not worth a
+// call that can fail.  Up to 8 lists the rank merge stays: it needs no bound.
 
 constexpr uint32_t kManyKept = 512;  // entries past the bound that are ranked
 
 // LDS of the selection, in the (then free) staging buffers.
 struct ManyLists {
-  uint64_t list[kMaxChunks * kMaxK];  // payloads, list c at c * 32 (kk <= 32) or c * 64
+  uint64_t list[kMaxChunks * kMaxK];  // composites, list c at c * 32 (kk <= 32) or c * 64
   uint64_t kept[kManyKept];
 };
 
-// The bound, by one wave (all lanes get it): at least kk payloads are >= it.
+// The bound, by one wave (all lanes get it): at least kk composites are >= it.
 //  * the kk-th largest, to 2^12 key units, of the lists' first m entries (m as
 //    many as 128 candidates hold, at least kk of them: two per lane, a ballot
 //    radix search over their keys);
@@ -1216,7 +1217,7 @@ __device__ __forceinline__ uint64_t many_bound(const uint64_t* list, uint32_t st
 #pragma unroll
   for (uint32_t h = 0; h < 2u; h++) {
     const uint32_t i = h * kWave + lane;
-    key[h] = i < n ? static_cast<uint32_t>(list[i % chunks * stride + i / chunks] >> kWireIdBits) : 0u;
+    key[h] = i < n ? comp_key(list[i % chunks * stride + i / chunks]) : 0u;
   }
   const uint64_t last = wave_max_u64(lane < chunks ? list[lane * stride + kk - 1u] : 0ull);
   uint32_t T = 0u;
@@ -1226,12 +1227,12 @@ __device__ __forceinline__ uint64_t many_bound(const uint64_t* list, uint32_t st
     if (static_cast<uint32_t>(__popcll(ballot(key[0] >= c)) + __popcll(ballot(key[1] >= c))) >= kk)
       T = c;
   }
-  const uint64_t floor = static_cast<uint64_t>(T) << kWireIdBits;
+  const uint64_t floor = static_cast<uint64_t>(T) << 31;
   return floor > last ? floor : last;
 }
 
 // The kk best of `chunks` lists in m.list (zeros past their ends and past kk)
-// as composites at out[rank] (zeroed by the caller).  All the workgroup's
+// at out[rank] (zeroed by the caller).  All the workgroup's
 // threads call; *kept (zeroed by the caller) counts the entries past the
 // bound.  Returns false, with nothing written, when they are more than are
 // ranked here.
@@ -1258,7 +1259,7 @@ __device__ __forceinline__ bool many_select(ManyLists& m, uint32_t stride, uint3
     const uint64_t e = m.kept[i];
     uint32_t r = 0u;
     for (uint32_t j = 0; j < n; j++) r += m.kept[j] > e ? 1u : 0u;
-    if (r < kk) out[r] = comp_of_payload(e);
+    if (r < kk) out[r] = e;
   }
   return true;
 }
@@ -1274,7 +1275,7 @@ namespace fg {
 template <class F>
 __global__ __launch_bounds__(kBlock, 3) void sample_rows_kernel(SampleArgs a) {
   __shared__ uint64_t s_buf[F::kTop ? kWaves : 1][F::kTop ? kCap + kWave : 1];
-  static_assert(!F::kTop || sizeof(s_buf) >= sizeof(ManyLists), "finisher lists in s_buf");
+  static_assert(!F::kTop || sizeof(s_buf) >= sizeof(ManyLists), "the chunks' lists in s_buf");
   __shared__ uint64_t s_top[kWaves][kWave];
   __shared__ uint64_t s_greedy[kWaves];
   __shared__ uint32_t s_ks[kWaves];
@@ -1285,10 +1286,10 @@ __global__ __launch_bounds__(kBlock, 3) void sample_rows_kernel(SampleArgs a) {
   __shared__ double s_ne[kWaves];
   __shared__ uint32_t s_wg_key;
   __shared__ uint64_t s_rank[kWave];
-  // A finisher of many chunks: the waves' speculative keys, the entries kept,
-  // whether some wave's wait gave up.
+  // The last of many chunks: the waves' speculative keys, the entries kept;
+  // whether this workgroup is it.
   __shared__ uint32_t s_ks_all[F::kMany && F::kSpec ? kMaxChunks * kWaves : 1];
-  __shared__ uint32_t s_kept, s_gave_up;
+  __shared__ uint32_t s_kept, s_last;
   FG_TRACE_DECL;
   FG_TRACE_INIT;
 
@@ -1436,22 +1437,23 @@ __global__ __launch_bounds__(kBlock, 3) void sample_rows_kernel(SampleArgs a) {
   if (F::kNuc && nuc) wmass = wave_mass_combine(static_cast<double>(st.nm), st.nz, st.ne);
 
   // ---- the workgroup's result: wave 0 combines the four waves from LDS ----
-  // Finisher protocol (top lists of at most 64 over 2-64 chunks, no
-  // log-probs or whole-row nucleus rows in the launch): one chunk finishes the
-  // row, reading the other chunks' lists until every entry carries the tag;
-  // the others store their lists tagged and end, with no wait for the stores
-  // and no arrival count (measured at config 2: 0.3 us less than the
-  // last-arriver hand-off; giving chunk 0 a longer slice, so that it would
-  // usually end last, cost more stream time than the wait it saved).  All four
-  // waves of the finishing workgroup rank the lists (up to 8) or select from
-  // them (more).
-  const bool fin_mode = F::kTop && !F::kLse && !F::kNuc && finisher_of(a) != 0u &&
-                        !greedy && kk != 0u && kk <= static_cast<uint32_t>(kMaxK);
+  // Finisher protocol (launches whose rows all keep top lists of at most 64
+  // over 2-8 chunks, nothing else): one chunk finishes the row, reading the
+  // other chunks' lists until every entry carries the tag; the others store
+  // their lists tagged and end, with no wait for the stores and no arrival
+  // count (measured at config 2: 0.3 us less than the last-arriver hand-off;
+  // giving chunk 0 a longer slice, so that it would usually end last, cost
+  // more stream time than the wait it saved).  All four waves of the
+  // finishing workgroup rank the lists.
+  const bool fin_mode = F::kTop && !F::kGreedy && !F::kLse && !F::kNuc && !F::kMany &&
+                        finisher_of(a) != 0u && kk != 0u && kk <= static_cast<uint32_t>(kMaxK);
   const bool fin_wg = fin_mode && a.chunks != 1u && chunk == finisher_of(a) - 1u;
-  // The same for greedy rows (no log-probs) over 2-64 chunks: one composite
-  // per chunk.
-  const bool gfin_mode = F::kGreedy && !F::kNuc && finisher_of(a) != 0u && greedy && L == 0u &&
+  // The same for batches of greedy rows (no log-probs) over 2-64 chunks:
+  // one composite per chunk.
+  const bool gfin_mode = F::kGreedy && !F::kTop && finisher_of(a) != 0u && L == 0u &&
                          a.chunks >= 2u && a.chunks <= static_cast<uint32_t>(kWave);
+  // Rows of more than 8 chunks: the last to arrive selects, with all its waves.
+  const bool many = F::kMany && !greedy;
   // The four waves rank their own lists' entries (five- or six-step
   // searches): lists of at most 32, and longer ones in launches without
   // whole-row nucleus or log-prob rows (there, one wave's bitonic merges
@@ -1513,13 +1515,30 @@ __global__ __launch_bounds__(kBlock, 3) void sample_rows_kernel(SampleArgs a) {
     }
   };
   if constexpr (F::kMany) {
-    if (fin_wg) {
+    if (many) {
+      const uint64_t row_slot = static_cast<uint64_t>(row) * a.chunks;
+      if (wave == 0) {
+        const uint64_t slot = row_slot + chunk;
+        if (lane < kk) store_coherent(a.cand + slot * kMaxK + lane, s_rank[lane]);
+        if (spec && lane < static_cast<uint32_t>(kWaves))
+          store_coherent(a.spec + slot * kWaves + lane, static_cast<uint64_t>(s_ks[lane]));
+        wait_memory();  // hand-off ordering: see wait_memory()
+        FG_TRACE(a, 3);
+        if (lane == 0) {
+          s_last = atomicAdd(&a.row_done[row * kLineWords], 1u) == a.chunks - 1u;
+          s_kept = 0u;
+        }
+        FG_TRACE(a, 4);
+      }
+      __syncthreads();  // every wave has left s_buf
+      if (!s_last) {
+        FG_TRACE_FLUSH(a);
+        return;
+      }
       // Wave w reads lists 16w .. 16w + 15 (lists of at most 32 two per
       // register, list 2t in lanes 0-31 and 2t + 1 in lanes 32-63 of x[t];
       // longer ones a register each), and its lane i the key of wave 64w + i.
       ManyLists& lists = *reinterpret_cast<ManyLists*>(&s_buf[0][0]);
-      const uint64_t row_slot = static_cast<uint64_t>(row) * a.chunks;
-      const uint64_t header = wire_header(a.finisher >> 16u);
       const bool wide = kk > 32u;
       const uint32_t stride = wide ? 64u : 32u;
       const uint32_t pos = lane & (stride - 1u);
@@ -1528,58 +1547,30 @@ __global__ __launch_bounds__(kBlock, 3) void sample_rows_kernel(SampleArgs a) {
         return 16u * wave + (wide ? t : 2u * t + (lane >> 5));
       };
       const uint32_t ks_i = static_cast<uint32_t>(kWave) * wave + lane;
-      const uint32_t ks_chunk = ks_i / static_cast<uint32_t>(kWaves);
-      uint64_t y = header;
-      auto fetch = [&]() {
-#pragma unroll
-        for (uint32_t t = 0; t < 16u; t++) {
-          const uint32_t c = list_of(t);
-          if ((wide || t < 8u) && c != chunk && c < a.chunks && pos < kk)
-            x[t] = load_coherent(a.cand + (row_slot + c) * kMaxK + pos);
-        }
-        if (spec && ks_chunk != chunk && ks_chunk < a.chunks)
-          y = load_coherent(a.spec + row_slot * kWaves + ks_i);
-      };
-#pragma unroll
-      for (uint32_t t = 0; t < 16u; t++) x[t] = header;
-      if (threadIdx.x == 0) s_kept = s_gave_up = 0u;
-      const uint64_t own = wire_payload(s_rank[lane]);
-      fetch();
-      bool late = false;
-      uint64_t t0 = 0ull;
-      for (uint32_t spin = 0;; spin++) {
-        bool miss = !wire_current(y, header);
-#pragma unroll
-        for (uint32_t t = 0; t < 16u; t++) miss |= !wire_current(x[t], header);
-        if (ballot(miss) == 0ull) break;
-        if (wait_passed(a, spin, t0)) {
-          late = true;
-          break;
-        }
-        __builtin_amdgcn_s_sleep(1);
-        fetch();
-      }
-      __syncthreads();  // every wave has its part of s_rank and has left s_buf
-      s_rank[lane] = 0ull;
-      if (late && lane == 0) s_gave_up = 1u;
+      const bool ks_read = spec && ks_i < a.chunks * static_cast<uint32_t>(kWaves);
 #pragma unroll
       for (uint32_t t = 0; t < 16u; t++) {
         const uint32_t c = list_of(t);
-        if ((wide || t < 8u) && c != chunk && c < a.chunks)
-          lists.list[c * stride + pos] = x[t] & kWirePayload;
+        x[t] = (wide || t < 8u) && c < a.chunks && pos < kk
+                   ? load_coherent(a.cand + (row_slot + c) * kMaxK + pos)
+                   : 0ull;
       }
-      if (wave == 0 && lane < stride) lists.list[chunk * stride + lane] = lane < kk ? own : 0ull;
+      const uint64_t y = ks_read ? load_coherent(a.spec + row_slot * kWaves + ks_i) : 0ull;
+      if (wave == 0) s_rank[lane] = 0ull;  // (read by this wave alone, above)
+#pragma unroll
+      for (uint32_t t = 0; t < 16u; t++) {
+        const uint32_t c = list_of(t);
+        if ((wide || t < 8u) && c < a.chunks) lists.list[c * stride + pos] = x[t];
+      }
       if constexpr (F::kSpec) {
-        if (spec && ks_chunk < a.chunks)
-          s_ks_all[ks_i] = ks_chunk == chunk ? s_ks[ks_i % kWaves] : static_cast<uint32_t>(y);
+        if (ks_read) s_ks_all[ks_i] = static_cast<uint32_t>(y);
       }
       __syncthreads();
       if (!many_select(lists, stride, a.chunks, kk, &s_kept, s_rank) && wave == 0) {
         // Too many past the bound (ties, crowded chunks): merged list by list.
         uint64_t best = 0ull;
         for (uint32_t c = 0; c < a.chunks; c++) {
-          const uint64_t e =
-              comp_of_payload(lane < kk ? lists.list[c * stride + (lane & (stride - 1u))] : 0ull);
+          const uint64_t e = lane < kk ? lists.list[c * stride + (lane & (stride - 1u))] : 0ull;
           if (readlane64(e, 0) > readlane64(best, kk - 1u)) best = wave_merge_desc(best, e);
         }
         s_rank[lane] = lane < kk ? best : 0ull;
@@ -1588,7 +1579,7 @@ __global__ __launch_bounds__(kBlock, 3) void sample_rows_kernel(SampleArgs a) {
     }
   }
   if (wave != 0) {
-    if (F::kTop && !F::kMany && fin_wg) {
+    if (F::kTop && fin_wg) {
       // The finisher's helpers: wave 0 fills the lists, all four rank them.
       __syncthreads();
       rank_place_lists(&s_top[0][0], &s_buf[0][0], wave, kk, a.chunks, s_rank);
@@ -1635,7 +1626,7 @@ __global__ __launch_bounds__(kBlock, 3) void sample_rows_kernel(SampleArgs a) {
     return;
   } else {
     const uint64_t slot = static_cast<uint64_t>(row) * a.chunks + chunk;
-    if (!fin_mode && !gfin_mode) {
+    if (!fin_mode && !gfin_mode && !many) {
       // Publish the workgroup's partials with device-coherent stores.
       if (F::kTop && kk && lane < kk) store_coherent(a.cand + slot * kMaxK + lane, fin);
       if (spec && lane < static_cast<uint32_t>(kWaves))
@@ -1667,10 +1658,10 @@ __global__ __launch_bounds__(kBlock, 3) void sample_rows_kernel(SampleArgs a) {
 
     // ---- last workgroup of the row: merge the other workgroups' lists ----
     const uint64_t row_slot = static_cast<uint64_t>(row) * a.chunks;
-    if (F::kMany && fin_mode) {
+    if (many) {
       // Selected by all four waves above.
       fin = lane < kk ? s_rank[lane] : 0ull;
-      gave_up = s_gave_up != 0u;
+      FG_TRACE(a, 5);
       if constexpr (F::kSpec) {
         if (spec) ks0 = spec_key(a, row, lane, ks_lds, ks_in_lds);
       }
@@ -1739,7 +1730,7 @@ __global__ __launch_bounds__(kBlock, 3) void sample_rows_kernel(SampleArgs a) {
               : ks_chunk < a.chunks ? static_cast<uint32_t>(y & kWirePayload) : 0u;
       }
       FG_TRACE(a, 5);
-    } else if (F::kTop && kk) {
+    } else if (F::kTop && !F::kMany && kk) {
       if (kk <= 32u) {
         // Lists of at most 32: two per register, the second loaded in
         // reverse into lanes 32-63, so a pair is already a bitonic sequence

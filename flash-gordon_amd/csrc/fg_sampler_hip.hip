@@ -505,17 +505,24 @@ fg_status sample_launch(const Workspace& w, const RowParams* h_params, uint32_t 
   a.split = geo.split;
   uint32_t finisher = 0u;
   {
-    // Finisher protocol (see the kernel): every row greedy or a top list of
-    // at most 64, no log-probs, over 2-64 chunks; ids that fit a tagged word.
-    // Not for a launch being captured into a graph: its replays would all
-    // carry the epoch it was captured with, so a word left by the previous
-    // replay would pass for the current one; the last-arriver hand-off keeps
-    // no state between launches.
+    // Finisher protocol (see the kernel): every row a top list of at most 64
+    // (no greedy row, no log-probs) over 2-8 chunks, or every row greedy (no
+    // log-probs) over 2-64 chunks; ids that fit a tagged word.  Not for a
+    // launch being captured into a graph: its replays would all carry the
+    // epoch it was captured with, so a word left by the previous replay
+    // would pass for the current one; the last-arriver hand-off keeps no
+    // state between launches.
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &capture) != hipSuccess) capture = hipStreamCaptureStatusNone;
+    bool all_greedy = true, any_greedy = false;
+    for (uint32_t r = 0; r < b->rows; r++) {
+      const bool greedy = h_params[r].temperature == 0.0f;
+      all_greedy &= greedy;
+      any_greedy |= greedy;
+    }
     const bool ok = capture == hipStreamCaptureStatusNone && w.tuning.finisher != 0 &&
-                    chunks >= 2u && chunks <= fg::kMaxChunks && b->logprobs == 0u && !nuc_rows &&
-                    vocab <= fg::kWireVocab;
+                    chunks >= 2u && b->logprobs == 0u && !nuc_rows && vocab <= fg::kWireVocab &&
+                    (all_greedy ? chunks <= fg::kMaxChunks : !any_greedy && chunks <= 8u);
     const uint32_t which = w.tuning.finisher > 0 ? static_cast<uint32_t>(w.tuning.finisher) - 1u : 0u;
     finisher = ok && which < chunks ? which + 1u : 0u;
   }
@@ -556,14 +563,14 @@ fg_status sample_launch(const Workspace& w, const RowParams* h_params, uint32_t 
                              fg::kSpecMaxElems;
   int bits = (any_pen ? 1 : 0) | (any_greedy ? 2 : 0) | (any_top ? 4 : 0) |
                    (b->logprobs ? 8 : 0) | (any_nuc ? 16 : 0) | (any_spec ? 32 : 0);
+  // More than 8 chunks a row: the last to arrive selects from all the lists.
+  if (any_top && chunks > 8u && !b->logprobs && !any_nuc) bits |= 64;
   const uint32_t grid = b->rows * chunks;
   // The finisher waits for the other workgroups of its row: only when the
   // whole grid fits on the device at once (occupancy x CUs) is every one of
   // them sure to run while it waits.  Otherwise the last arriver finishes.
-  const int fin_bits = any_top && chunks > 8u ? bits | 64 : bits;
   if (finisher && static_cast<uint64_t>(grid) <=
-                      static_cast<uint64_t>(occupancy(fin_bits)) * w.cus) {
-    bits = fin_bits;
+                      static_cast<uint64_t>(occupancy(bits)) * w.cus) {
     uint32_t epoch = 0u;
     const hipError_t e = next_epoch(w, stream, &epoch);
     if (e != hipSuccess) return hip_fail(err, e, "sampler epoch");

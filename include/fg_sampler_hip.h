@@ -170,7 +170,8 @@ void fg_sampler_hip_destroy(fg_sampler_hip *sampler);
  * later fg_sampler_hip_sample calls, in microseconds (default 100000).  In
  * that hand-off one workgroup of each row waits, on the device, for the
  * row's other workgroups (it is used only when the whole launch fits on the
- * device at once); a row whose wait passes the limit gets row_status
+ * device at once, for batches of greedy rows and for batches of top-k rows
+ * over at most 8 workgroups each; any other batch waits for nobody); a row whose wait passes the limit gets row_status
  * FG_ERR_UNAVAILABLE and token 0xffffffff instead of a token.  0 makes
  * every such row that is not complete at the first look report it (a
  * host-side way to exercise that path). */
