@@ -780,6 +780,10 @@ fg_status fg_hip_output_slice_create(fg_hip_output_slice** out, uint32_t vocab, 
         fg_hip_output_slice_destroy(s);
         return st;
       }
+      // The last-arriver hand-off alone: it waits for nobody, so no token of a
+      // sampled call can miss a wait limit (beside the product, what the
+      // tagged one saves at 64 tokens is lost: 0.3 of 310 us).
+      s->sampler->ws.tuning.finisher = 0;
     }
     if (e == hipSuccess) e = hipDeviceSynchronize();
   }

@@ -94,6 +94,29 @@ def test_sampled_lm_head_matches_unfused(dev, vocab, width, tokens, scale):
     assert np.array_equal(got["logit"][same].view(np.uint32), ref["logit"][same].view(np.uint32))
 
 
+@pytest.mark.parametrize("tokens", [1, 3, 64])
+@pytest.mark.parametrize("kind", ["greedy", "top-k", "mixed"])
+def test_sampled_lm_head_waits_for_nobody(dev, monkeypatch, tokens, kind):
+    """A wait limit of 0, as the environment gives it at create, fails no token."""
+    import torch
+    monkeypatch.setenv("FG_HIP_FINISHER_WAIT_US", "0")
+    vocab, width = 100_003, 64
+    rng = np.random.default_rng(tokens)
+    cooked = torch.from_numpy(cooked_random(rng, width, vocab)).to(dev)
+    hidden = torch.from_numpy(rng.normal(0, 1, (tokens, width)).astype(np.float32)).to(dev)
+    controls = {"greedy": [(0.0, 1.0, 1)], "top-k": [(0.7, 0.9, 20)],
+                "mixed": [(0.0, 1.0, 1), (0.7, 0.9, 20)]}[kind]
+    configs = [fg_hip.make_config(*controls[t % len(controls)]) for t in range(tokens)]
+    uniforms = torch.from_numpy(rng.random(tokens).astype(np.float32)).to(dev)
+    sl = fg_hip.OutputSlice(vocab, 1, 0, vocab, tokens)
+    tok, st = (torch.full((tokens,), -7, dtype=torch.int32, device=dev) for _ in range(2))
+    lg = torch.empty(tokens, device=dev)
+    for _ in range(3):
+        sl.run_dense_sampled(cooked, hidden, width, tokens, configs, uniforms, tok, lg, st, scale=0.1)
+        assert not st.any().item()
+        assert ((tok >= 0) & (tok < vocab)).all().item()
+
+
 @pytest.mark.parametrize("kind", ["zero_input", "nan_input", "inf_scale_row", "tied_rows"])
 def test_sampled_lm_head_special_values(dev, kind):
     """Zero logits (either sign), NaN and infinite logits, and ties, for
