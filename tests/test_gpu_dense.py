@@ -43,7 +43,7 @@ def plain(dev, cooked, x, width, rows, scale):
     return y.cpu().numpy().reshape(tokens, rows)
 
 
-def check_f64(y, packed, x, width, rows, scale, sample=None):
+def check_f64(y, packed, x, width, rows, scale, sample=None, floor=1e-30):
     if sample is not None:
         blocks = width // 32
         sub = packed.reshape(rows, blocks * 34)[sample].reshape(-1)
@@ -52,8 +52,8 @@ def check_f64(y, packed, x, width, rows, scale, sample=None):
     else:
         want, mag = O.dense_q8_0_f64(packed, x, width, rows, scale)
     err = np.abs(y.astype(np.float64) - want)
-    assert np.all(err <= TOL * mag + 1e-30), float(np.max(err / (mag + 1e-30)))
-    return float(np.max(err / (mag + 1e-30)))
+    assert np.all(err <= TOL * mag + floor), float(np.max(err / (mag + floor)))
+    return float(np.max(err / (mag + floor)))
 
 
 def test_reference_cooked_dense_case(dev):

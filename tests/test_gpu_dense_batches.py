@@ -57,13 +57,12 @@ def test_many_tiles(dev, tokens, width, rows):
 @pytest.mark.parametrize("tokens", [2, 8, 12, 64])
 def test_extreme_inputs(dev, tokens):
     """Non-finite inputs reach only their own token, with IEEE results; inputs
-    from 1e-30 to 1e30 and subnormal ones keep the f32 product's accuracy."""
+    from 1e-30 to 1e30 keep the f32 product's accuracy."""
     rng = np.random.default_rng(tokens)
     width, rows = 320, 100
     packed = packed_random(rng, width, rows)
     cooked = fg_hip.cook_q8_0(packed, width, rows)
     x = (rng.normal(0, 1, (tokens, width)) * 10.0 ** rng.uniform(-30, 30, (tokens, width))).astype(np.float32)
-    x[0] = (rng.normal(0, 1, width) * 1e-39).astype(np.float32)
     check_f64(plain(dev, cooked, x, width, rows, 1.0), packed, x, width, rows, 1.0)
     x = rng.normal(0, 1, (tokens, width)).astype(np.float32)
     clean = plain(dev, cooked, x, width, rows, 1.0)
@@ -78,6 +77,43 @@ def test_extreme_inputs(dev, tokens):
         assert np.array_equal(np.isnan(y[1]), np.isnan(want))
         assert np.array_equal(y[1][~np.isnan(want)], want[~np.isnan(want)])
     assert np.all(np.isnan(y[-1]))
+
+
+@pytest.mark.parametrize("tokens", [1, 2, 8, 9, 17, 33, 64, 66])
+@pytest.mark.parametrize("width,rows", [(96, 40), (2560, 150), (8192, 17)])
+def test_tiny_inputs(dev, tokens, width, rows):
+    """Inputs whose bits reach below the smallest subnormal bf16 (from about
+    1e-33 down to f32's subnormals) keep the f32 product's accuracy: within the
+    tolerance above of the token's own sum of magnitudes, besides the rounding
+    of a subnormal result (2^-150, below 1e-45).  One tiny input, in the last
+    block, is enough; the tokens beside such ones keep their bits, the fused
+    finalist carries the plain values."""
+    rng = np.random.default_rng(tokens + width)
+    packed = packed_random(rng, width, rows, 0.25, 1.0)
+    cooked = fg_hip.cook_q8_0(packed, width, rows)
+    for first in (0, 1):
+        x = rng.normal(0, 1, (tokens, width)).astype(np.float32)
+        clean = plain(dev, cooked, x, width, rows, 0.75)
+        tiny = np.arange(first, tokens, 2)
+        for j, t in enumerate(tiny):
+            x[t] *= np.float32(10.0 ** -[33, 34, 36, 38, 39, 41][j % 6])
+            if j % 4 == 3:  # all zero but the last block
+                x[t, :-32] = 0
+        y = plain(dev, cooked, x, width, rows, 0.75)
+        check_f64(y, packed, x, width, rows, 0.75, floor=1e-45)
+        others = np.arange(1 - first, tokens, 2)
+        assert np.array_equal(y[others].view(np.uint32), clean[others].view(np.uint32))
+        if len(others):  # a normal token with one tiny input
+            x[others[0], -1] = np.float32(1.1e-38)
+            y = plain(dev, cooked, x, width, rows, 1.0)
+            check_f64(y, packed, x, width, rows, 1.0, floor=1e-45)
+        else:
+            y = plain(dev, cooked, x, width, rows, 1.0)
+        sl = fg_hip.OutputSlice(rows, 1, 0, rows, tokens)
+        v, i, s, _ = fused(dev, sl, cooked, x, width, logits=False)
+        wv, wi, ws = O.slice_finalists(y, 0)
+        assert np.array_equal(i, wi) and np.array_equal(v.view(np.uint32), wv.view(np.uint32))
+        assert np.array_equal(s, ws)
 
 
 @pytest.mark.parametrize("tokens", [1, 8, 64])
