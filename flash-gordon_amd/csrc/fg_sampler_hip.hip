@@ -117,7 +117,7 @@ template <class S, bool kFused>
 hipError_t dense_pass(fg::DenseArgs a, hipStream_t stream) {
   const uint32_t per = S::kR * S::kWV;
   const uint32_t groups = (dense_tiles(a.rows) + per - 1u) / per;
-  const uint32_t body = S::kBody, blocks = (a.in / 32u + body - 1u) / body * body;
+  const uint32_t body = fg::kDenseBody, blocks = (a.in / 32u + body - 1u) / body * body;
   a.slice = std::min(S::slice(a.tokens), blocks);
   const uint32_t lds = a.slice * S::block_bytes(a.tokens) * (blocks > a.slice ? 2u : 1u);
   const void* k = reinterpret_cast<const void*>(&fg::dense_q8_kernel<S, kFused>);
@@ -130,45 +130,82 @@ hipError_t dense_pass(fg::DenseArgs a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// Tiles of the CU with most of them, at `per` a workgroup.
+uint32_t dense_load(uint32_t tiles, uint32_t per) {
+  const uint32_t groups = (tiles + per - 1u) / per;
+  return (groups + fg::kDenseCus - 1u) / fg::kDenseCus * per;
+}
+
 // The pass's shape, by the call's tokens (the form, fg_dense_kernels.hpp) and
-// the pass's (248,320 x 2,560: 111 us at 1 token, 113 at 2, 116 at 5, 129 at
-// 8, 132 at 16, 186 at 32, 300 at 64; the vector kernel this replaces took 107,
-// 124, -, 488, -, -, 3,810: its order of sums cannot be kept for one token
-// alone, whose bits are those of any call up to 8), then by the matrix: more rows a wave and more
-// waves a workgroup share more of the staging and of the operand reads, down
-// to matrices that no longer give 7 of 8 CUs a workgroup (32,000 rows of
-// 2,560, the next smaller shape against the larger: 33 against 40 us at 32
-// tokens, 51 against 66 at 64; 62,080 rows: 52 against 48 and 99 against 74).
-// Up to 5 tokens little is shared, and what counts is how evenly the
-// workgroups fill the CUs (100,000 rows, one token: 46 us at one tile a wave,
-// 49 at two; 248,320: 103 at both).
-template <bool kFused, bool kLines>
-hipError_t dense_shape(const fg::DenseArgs& a, uint32_t call_tokens, hipStream_t stream) {
+// the pass's, then by the matrix: two tiles a wave and eight waves a workgroup
+// share more of the operand reads and of the staging, as far as the
+// workgroups still fill the CUs evenly.  Measured, us:
+//   * up to 5 tokens, where little is shared: two tiles a wave (1 token at
+//     248,320 x 2,560 103, at 50,355 x 6,944 65; one tile 100 and 73, but 116
+//     against 110 at 4 tokens), one if that leaves the fullest CU 1/16 less to
+//     do (100,000 x 2,560: 46, two 50; 43,428 x 4,032: 34 and 40) or all fit
+//     one round of workgroups (32,000 x 2,560: 17.3 and 18.0);
+//   * 6 to 8: the same, eight waves as long as the CUs get one workgroup each
+//     (8 tokens at 32,000 x 2,560: 19.8, four waves 21.6; 50,355 x 6,944: 80
+//     and 87), then four (248,320 x 2,560: 125, in eight 133);
+//   * 9 to 16: two tiles, in eight waves if that leaves the CUs as even as
+//     four (100,000 x 2,560: 61, in four 66; 132,576 x 3,104: 126 and 113), or
+//     four tiles in four for more than 8,192 (248,320 x 2,560: 133, two tiles
+//     in eight 138; past that the registers of the shifted stream spill);
+//   * more: two tiles in eight waves (248,320 x 2,560: 189 at 32 tokens, 246 at
+//     48, 296 at 64; one tile 224, 305, 393), less below 2,048 and 1,024 tiles.
+template <bool kFused, fg::DenseRows kRows>
+hipError_t dense_to_16(const fg::DenseArgs& a, uint32_t call_tokens, hipStream_t stream) {
   using fg::DenseShape;
-  constexpr uint32_t kMostCus = 224u;
+  constexpr bool kShift = kRows == fg::kShifted;
   const uint32_t tiles = dense_tiles(a.rows);
-  const bool large = tiles >= 16u * kMostCus, middle = tiles >= 8u * kMostCus;
-  if (call_tokens <= 5u)
-    return tiles >= 8192u ? dense_pass<DenseShape<false, 1, 2, 4, 2, 2, 3, kLines>, kFused>(a, stream)
-                          : dense_pass<DenseShape<false, 1, 1, 4, 2, 2, 4, kLines>, kFused>(a, stream);
-  if (call_tokens <= fg::kDenseSideBySide)
-    return large ? dense_pass<DenseShape<false, 2, 2, 4, 1, 2, 3, kLines>, kFused>(a, stream)
-                 : dense_pass<DenseShape<false, 2, 1, 4, 2, 2, 4, kLines>, kFused>(a, stream);
-  if (a.tokens <= 16u)
-    return large    ? dense_pass<DenseShape<true, 1, 4, 4, 1, 2, 2, kLines>, kFused>(a, stream)
-           : middle ? dense_pass<DenseShape<true, 1, 2, 4, 2, 2, 3, kLines>, kFused>(a, stream)
-                    : dense_pass<DenseShape<true, 1, 1, 4, 2, 2, 4, kLines>, kFused>(a, stream);
+  const uint32_t four = dense_load(tiles, 4u), eight = dense_load(tiles, 8u);
+  const bool few = tiles <= 4u * fg::kDenseCus, some = tiles <= 8u * fg::kDenseCus;
+  const bool one = eight * 15u > four * 16u;
+  if (call_tokens <= 5u) {
+    if (some || one)
+      return dense_pass<DenseShape<false, 1, 1, 4, 2, 2, kShift ? 3 : 4, kRows>, kFused>(a, stream);
+    return dense_pass<DenseShape<false, 1, 2, 4, kShift ? 1 : 2, 2, kShift ? 3 : 2, kRows>, kFused>(
+        a, stream);
+  }
+  if (call_tokens <= fg::kDenseSideBySide) {
+    if (some && !few)
+      return dense_pass<DenseShape<false, 2, 1, 8, 2, 2, 3, kRows>, kFused>(a, stream);
+    if (few || one)
+      return dense_pass<DenseShape<false, 2, 1, 4, 2, 2, 3, kRows>, kFused>(a, stream);
+    if (tiles <= 16u * fg::kDenseCus)
+      return dense_pass<DenseShape<false, 2, 2, 8, 2, 2, 2, kRows>, kFused>(a, stream);
+    constexpr int kDeep = kShift ? 2 : 1;  // steps ahead, units a thread
+    return dense_pass<DenseShape<false, 2, 2, 4, kDeep, kDeep, kShift ? 2 : 3, kRows>, kFused>(
+        a, stream);
+  }
+  if (few)
+    return dense_pass<DenseShape<true, 1, 1, 4, 2, 2, kShift ? 3 : 4, kRows>, kFused>(a, stream);
+  if (some) return dense_pass<DenseShape<true, 1, 1, 8, 2, 2, 3, kRows>, kFused>(a, stream);
+  if constexpr (!kShift)
+    if (tiles > 32u * fg::kDenseCus && dense_load(tiles, 16u) <= eight)
+      return dense_pass<DenseShape<true, 1, 4, 4, 1, 2, 2, kRows>, kFused>(a, stream);
+  return dense_load(tiles, 16u) <= eight
+             ? dense_pass<DenseShape<true, 1, 2, 8, 2, 2, 2, kRows>, kFused>(a, stream)
+             : dense_pass<DenseShape<true, 1, 2, 4, 2, 2, 2, kRows>, kFused>(a, stream);
+}
+
+template <bool kFused, fg::DenseRows kRows>
+hipError_t dense_past_16(const fg::DenseArgs& a, hipStream_t stream) {
+  using fg::DenseShape;
+  const uint32_t tiles = dense_tiles(a.rows);
+  const bool few = tiles <= 4u * fg::kDenseCus, some = tiles <= 8u * fg::kDenseCus;
   if (a.tokens <= 32u)
-    return large    ? dense_pass<DenseShape<true, 2, 2, 8, 1, 2, 2, kLines>, kFused>(a, stream)
-           : middle ? dense_pass<DenseShape<true, 2, 2, 4, 1, 2, 2, kLines>, kFused>(a, stream)
-                    : dense_pass<DenseShape<true, 2, 1, 4, 2, 2, 3, kLines>, kFused>(a, stream);
+    return few    ? dense_pass<DenseShape<true, 2, 1, 4, 2, 2, 3, kRows>, kFused>(a, stream)
+           : some ? dense_pass<DenseShape<true, 2, 1, 8, 1, 2, 3, kRows>, kFused>(a, stream)
+                  : dense_pass<DenseShape<true, 2, 2, 8, 1, 2, 2, kRows>, kFused>(a, stream);
   if (a.tokens <= 48u)
-    return large    ? dense_pass<DenseShape<true, 3, 2, 8, 1, 3, 2, kLines>, kFused>(a, stream)
-           : middle ? dense_pass<DenseShape<true, 3, 1, 8, 1, 3, 2, kLines>, kFused>(a, stream)
-                    : dense_pass<DenseShape<true, 3, 1, 4, 1, 3, 2, kLines>, kFused>(a, stream);
-  return large    ? dense_pass<DenseShape<true, 4, 2, 8, 2, 2, 2, kLines>, kFused>(a, stream)
-         : middle ? dense_pass<DenseShape<true, 4, 1, 8, 2, 2, 2, kLines>, kFused>(a, stream)
-                  : dense_pass<DenseShape<true, 4, 1, 4, 2, 4, 2, kLines>, kFused>(a, stream);
+    return few    ? dense_pass<DenseShape<true, 3, 1, 4, 1, 3, 2, kRows>, kFused>(a, stream)
+           : some ? dense_pass<DenseShape<true, 3, 1, 8, 2, 3, 2, kRows>, kFused>(a, stream)
+                  : dense_pass<DenseShape<true, 3, 2, 8, 1, 3, 2, kRows>, kFused>(a, stream);
+  return few    ? dense_pass<DenseShape<true, 4, 1, 4, 2, 4, 2, kRows>, kFused>(a, stream)
+         : some ? dense_pass<DenseShape<true, 4, 1, 8, 2, 2, 2, kRows>, kFused>(a, stream)
+                : dense_pass<DenseShape<true, 4, 2, 8, 2, 2, 2, kRows>, kFused>(a, stream);
 }
 
 // `tokens` of a call of `call_tokens` from a.token0 = 0 on, in passes.
@@ -178,8 +215,13 @@ hipError_t dense_launch(fg::DenseArgs a, uint32_t tokens, uint32_t call_tokens,
   for (uint32_t t0 = 0; t0 < tokens; t0 += fg::kDensePassTokens) {
     a.token0 = t0;
     a.tokens = std::min(tokens - t0, fg::kDensePassTokens);
-    const hipError_t e = a.in % 128u == 0u ? dense_shape<kFused, true>(a, call_tokens, stream)
-                                           : dense_shape<kFused, false>(a, call_tokens, stream);
+    const bool on = a.in % 128u == 0u;
+    const hipError_t e =
+        a.tokens <= 16u
+            ? (on ? dense_to_16<kFused, fg::kOnLines>(a, call_tokens, stream)
+                  : dense_to_16<kFused, fg::kShifted>(a, call_tokens, stream))
+            : (on ? dense_past_16<kFused, fg::kOnLines>(a, stream)
+                  : dense_past_16<kFused, fg::kOffLines>(a, stream));
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

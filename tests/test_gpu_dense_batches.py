@@ -1,6 +1,7 @@
 """The Q8_0 product at the edges of its shapes: every count of tokens where the
-form or the column tiles change, widths that leave partial steps and slices,
-matrices of few and of many tiles, non-finite inputs.
+columns held or the column tiles change, widths that leave partial steps and
+slices or whose rows start off the cache lines, matrices of few and of many
+tiles, non-finite and tiny inputs.
 
 Tolerance: an output sums exact products in f32: within 1e-6 of the sum of
 magnitudes of the f64 product (24 roundings of 2^-24 at the widest row are
@@ -16,7 +17,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("tokens", [1, 2, 5, 6, 8, 9, 16, 17, 32, 33, 48, 49, 64, 65, 130])
-@pytest.mark.parametrize("width,rows", [(96, 40), (2560, 300), (8192, 17)])
+@pytest.mark.parametrize("width,rows", [(32, 16), (96, 40), (160, 300), (192, 33), (2560, 300),
+                                        (6944, 50), (8192, 17)])
 def test_tokens_widths(dev, tokens, width, rows):
     rng = np.random.default_rng(tokens * 31 + width)
     packed = packed_random(rng, width, rows)
@@ -30,16 +32,15 @@ def test_tokens_widths(dev, tokens, width, rows):
     wv, wi, ws = O.slice_finalists(ref, 0)
     assert np.array_equal(i, wi) and np.array_equal(v.view(np.uint32), wv.view(np.uint32))
     assert np.array_equal(s, ws)
-    # A token's logits are the same beside any others of its form.
-    form = tokens <= 8
-    less = [n for n in (1, 3, 7, 9, 20, 50) if n < tokens and (n <= 8) == form]
-    for n in less:
+    # A token's logits have the same bits beside any others of its form.
+    for n in (m for m in (1, 3, 6, 8, 9, 16, 17, 50) if m < tokens and (m <= 8) == (tokens <= 8)):
         assert np.array_equal(plain(dev, cooked, x[:n], width, rows, 1.0).view(np.uint32),
                               ref[:n].view(np.uint32)), n
 
 
-@pytest.mark.parametrize("tokens", [1, 7, 16, 30, 40, 64])
-@pytest.mark.parametrize("width,rows", [(32, 29_001), (64, 57_345), (288, 131_073), (2_176, 28_672)])
+@pytest.mark.parametrize("tokens", [1, 4, 7, 16, 30, 40, 64])
+@pytest.mark.parametrize("width,rows", [(32, 29_001), (64, 57_345), (160, 127_990), (256, 70_001),
+                                        (256, 127_990), (288, 131_073), (2_176, 28_672)])
 def test_many_tiles(dev, tokens, width, rows):
     rng = np.random.default_rng(tokens + width)
     packed = packed_random(rng, width, rows)
@@ -52,6 +53,28 @@ def test_many_tiles(dev, tokens, width, rows):
     v, i, s, _ = fused(dev, sl, cooked, x, width, logits=False)
     wv, wi, ws = O.slice_finalists(y, 0)
     assert np.array_equal(i, wi) and np.array_equal(v.view(np.uint32), wv.view(np.uint32))
+    # The bits of the form's fewest tokens (another shape).
+    n = 1 if tokens <= 8 else 9
+    assert np.array_equal(plain(dev, cooked, x[:n], width, rows, 1.0).view(np.uint32),
+                          y[:n].view(np.uint32))
+
+
+@pytest.mark.parametrize("width,rows", [(32, 3), (96, 700), (160, 131_073), (6944, 33)])
+def test_weights_off_the_lines(dev, width, rows):
+    """Weights 16-byte aligned but not on a cache line: the same bits."""
+    import torch
+    rng = np.random.default_rng(width)
+    packed = packed_random(rng, width, rows)
+    cooked = fg_hip.cook_q8_0(packed, width, rows)
+    x = rng.normal(0, 1, (3, width)).astype(np.float32)
+    want = plain(dev, cooked, x, width, rows, 1.0)
+    for at in (16, 80):
+        buf = torch.zeros(len(cooked) + 128, dtype=torch.uint8, device=dev)
+        w = buf[at:at + len(cooked)]
+        w.copy_(torch.from_numpy(cooked))
+        y = torch.empty(3 * rows, dtype=torch.float32, device=dev)
+        fg_hip.dense_q8_0_cooked(y, w, torch.from_numpy(x).to(dev), width, rows, 3, 1.0)
+        assert np.array_equal(y.cpu().numpy().view(np.uint32).reshape(3, rows), want.view(np.uint32))
 
 
 @pytest.mark.parametrize("tokens", [2, 8, 12, 64])
