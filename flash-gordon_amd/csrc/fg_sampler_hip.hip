@@ -770,8 +770,9 @@ struct fg_hip_output_slice {
 };
 
 // The sampled output's logits workspace holds at most this many bytes (one
-// token's logits at least).
-constexpr uint64_t kSampleLogitsBytes = 256ull << 20;
+// token's logits at least): 64 tokens of up to 262,144 ids.  Every whole-head
+// slice allocates it, so that no call has to.
+constexpr uint64_t kSampleLogitsBytes = 64ull << 20;
 
 fg_status fg_hip_output_slice_create(fg_hip_output_slice** out, uint32_t vocab, uint32_t ways,
                                      uint32_t first_row, uint32_t rows,
@@ -815,7 +816,14 @@ fg_status fg_hip_output_slice_create(fg_hip_output_slice** out, uint32_t vocab, 
     s->sample_tokens = static_cast<uint32_t>(std::max<uint64_t>(
         1u, std::min<uint64_t>(std::min(max_batch_rows, fg::kDensePassTokens),
                                kSampleLogitsBytes / row_bytes)));
-    if (e == hipSuccess) e = hipMalloc(&s->d_logits, row_bytes * s->sample_tokens);
+    // Short of memory, fewer tokens a pass will do.
+    while (e == hipSuccess) {
+      const hipError_t got = hipMalloc(&s->d_logits, row_bytes * s->sample_tokens);
+      if (got == hipSuccess) break;
+      (void)hipGetLastError();
+      if (s->sample_tokens == 1u) e = got;
+      s->sample_tokens /= 2u;
+    }
     if (e == hipSuccess) {
       const fg_status st = fg_sampler_hip_create(&s->sampler, vocab, s->sample_tokens, err);
       if (st != FG_OK) {

@@ -385,8 +385,9 @@ fg_status fg_hip_output_slice_run_dense(fg_hip_output_slice *slice, const void *
  * 0, rows == vocab); configs are host memory, validated as
  * fg_sampler_config_validate does (FG_ERR_ARGUMENT, "invalid sampler
  * controls").  Two launches per pass of up to 64 tokens (the product, then
- * the sampler over its logits, which stay in the slice's workspace: 256 MB at
- * most, allocated at create).  Nothing in it waits for another workgroup, so
+ * the sampler over its logits, which stay in the slice's workspace: 64 MB at
+ * most, allocated at create; wider vocabularies take fewer tokens a pass, and
+ * so does a slice created when memory is short).  Nothing in it waits for another workgroup, so
  * row_status is never FG_ERR_UNAVAILABLE.  Calls on one slice must not
  * overlap.  The history increment stays a separate step
  * (fg_sampler_hip_history_increment, or the caller's own). */

@@ -1,5 +1,6 @@
-"""A new sampler's hand-off workspace carries no word of an earlier one, on the
-CPU: tests/c/test_workspace_create.c stands in for the HIP calls of create."""
+"""What a new sampler and a new output slice leave in and take of device memory,
+on the CPU: tests/c/test_workspace_create.c stands in for the HIP calls of
+create."""
 import subprocess
 from pathlib import Path
 
@@ -23,4 +24,11 @@ def program(tmp_path_factory):
 
 def test_hand_off_words_start_cleared(program):
     r = subprocess.run([program], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_slice_workspace(program):
+    """A whole-head slice holds 64 tokens' logits in 64 MB at most, and takes
+    fewer when memory is short."""
+    r = subprocess.run([program, "slice"], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
