@@ -4,8 +4,12 @@ slices or whose rows start off the cache lines, matrices of few and of many
 tiles, non-finite and tiny inputs.
 
 Tolerance: an output sums exact products in f32: within 1e-6 of the sum of
-magnitudes of the f64 product (24 roundings of 2^-24 at the widest row are
-below 1.5e-6 of it in the worst case; observed errors are below 2e-8)."""
+magnitudes of the f64 product (at most 8 + 8 + 4 sums, two roundings a block
+and the scale's, each of 2^-24 of a partial sum: 1.4e-6 of it if every partial
+sum were the whole).  Wide rows of random signs hold to 1e-7: their partial
+sums stay below 5 sqrt(n) of n terms, a ninth of the magnitudes at 2,560
+inputs, and some 20 independent roundings of that add to 1.5e-8 rms; a lost
+low part would give 6e-7 at 8,192 inputs."""
 import numpy as np
 import pytest
 
@@ -25,7 +29,8 @@ def test_tokens_widths(dev, tokens, width, rows):
     cooked = fg_hip.cook_q8_0(packed, width, rows)
     x = rng.normal(0, 1, (tokens, width)).astype(np.float32)
     y = plain(dev, cooked, x, width, rows, 0.75)
-    check_f64(y, packed, x, width, rows, 0.75)
+    worst = check_f64(y, packed, x, width, rows, 0.75)
+    assert width < 2560 or worst <= 1e-7
     sl = fg_hip.OutputSlice(rows, 1, 0, rows, tokens)
     ref = plain(dev, cooked, x, width, rows, 1.0)
     v, i, s, _ = fused(dev, sl, cooked, x, width, logits=False)
@@ -57,6 +62,32 @@ def test_many_tiles(dev, tokens, width, rows):
     n = 1 if tokens <= 8 else 9
     assert np.array_equal(plain(dev, cooked, x[:n], width, rows, 1.0).view(np.uint32),
                           y[:n].view(np.uint32))
+
+
+@pytest.mark.parametrize("tokens", [1, 5, 8, 9, 16, 33, 64])
+@pytest.mark.parametrize("width,rows", [(96, 40), (2560, 64), (6944, 20), (8192, 17)])
+def test_low_parts_decide(dev, tokens, width, rows):
+    """Inputs in pairs that differ in their lowest 8 bits alone, against weights
+    that cancel the rest, in one block at a time: what is left is the low parts'
+    sum, about 4e-6 of the magnitudes, so that one lost in any slice shows."""
+    rng = np.random.default_rng(tokens * 7 + width)
+    blocks = width // 32
+    b = packed_random(rng, width, rows).reshape(rows, blocks, 34)
+    q = rng.integers(1, 128, (rows, blocks, 16), dtype=np.int8)
+    b[:, :, 2::2] = q.view(np.uint8)
+    b[:, :, 3::2] = (-q).view(np.uint8)
+    packed = b.reshape(-1)
+    cooked = fg_hip.cook_q8_0(packed, width, rows)
+    for at in np.unique([0, blocks // 3, blocks // 2, blocks - 2, blocks - 1]):
+        base = np.uint32(0x3f800000) | rng.integers(0, 1 << 15, (tokens, 16), dtype=np.uint32) << 8
+        x = np.zeros((tokens, width), dtype=np.float32)
+        x[:, 32 * at + 1:32 * at + 32:2] = base.view(np.float32)
+        x[:, 32 * at:32 * at + 32:2] = (
+            base | rng.integers(64, 256, (tokens, 16), dtype=np.uint32)).view(np.float32)
+        y = plain(dev, cooked, x, width, rows, 1.0)
+        want, mag = O.dense_q8_0_f64(packed, x, width, rows, 1.0)
+        assert np.all(want > 3e-6 * mag)
+        assert np.all(np.abs(y - want) <= 1e-7 * mag), (at, np.max(np.abs(y - want) / mag))
 
 
 @pytest.mark.parametrize("width,rows", [(32, 3), (96, 700), (160, 131_073), (6944, 33)])

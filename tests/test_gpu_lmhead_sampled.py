@@ -1,13 +1,13 @@
 """GPU parity of the sampled LM head (fg_hip_output_slice_run_dense_sampled:
-the Q8_0 product fused with penalties, the top-k ladder and the select,
-src/output.c:702-756) against the unfused path on the same inputs: the plain
-product's logits (fg_hip_dense_q8_0_cooked) sampled by fg_sampler_hip_sample,
-which must agree bit for bit (token, logit bits, status), and sampled by the
-C oracle on the host, which must agree under the north-star bar (token ids
-bit-exact unless the oracle's draw lies within 1e-6 of a boundary, logits
-bit-exact where the tokens agree).  Vocabularies of 4,099 (a partial tile,
-one merge group), 151,936 (38 groups) and the reference's 248,320 x 2,560
-head (61 groups); greedy rows with and without penalties, top-k 1..64."""
+the Q8_0 product, then penalties, the top-k ladder and the select,
+src/output.c:702-756) against the plain product's logits
+(fg_hip_dense_q8_0_cooked) sampled by fg_sampler_hip_sample, which must agree
+bit for bit (token, logit bits, status), and sampled by the C oracle on the
+host, which must agree on the token ids bit for bit unless the oracle's draw
+lies within 1e-6 of a boundary, and on the logits bit for bit where the tokens
+agree.  Vocabularies of 4,099 (a partial tile), 151,936, 600,001 (few tokens
+a pass) and the reference's 248,320 x 2,560 head; one pass and several;
+greedy rows with and without penalties, top-k 1..64."""
 import numpy as np
 import pytest
 
@@ -76,7 +76,9 @@ def run_both(dev, cooked, hidden, width, vocab, configs, counts_np, uniforms_np,
 
 
 @pytest.mark.parametrize("vocab,width,tokens,scale", [(4099, 64, 3, 0.5), (151_936, 512, 6, 0.1),
-                                                      (248_320, 2560, 4, 0.05)])
+                                                      (248_320, 2560, 4, 0.05), (4099, 96, 9, 0.5),
+                                                      (20_000, 160, 64, 0.3), (4099, 64, 65, 0.5),
+                                                      (4099, 96, 130, 0.5), (600_001, 32, 60, 0.5)])
 def test_sampled_lm_head_matches_unfused(dev, vocab, width, tokens, scale):
     import torch
     rng = np.random.default_rng(vocab + width)

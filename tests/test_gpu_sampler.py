@@ -642,17 +642,18 @@ def test_finisher_wait_limit_reports_and_next_call_is_exact(dev, greedy):
         check(w2, run_hip(w2, dev, sampler=s), W.oracle_run(w2), f"after the limit, call {call}")
 
 
-def test_finisher_epoch_wrap(dev, monkeypatch):
+@pytest.mark.parametrize("top_k", [16, 50])
+def test_finisher_epoch_wrap(dev, monkeypatch, top_k):
     """The hand-off epoch runs 1..8191 and the workspace is cleared when it
     wraps: 8,200 calls of a two-row batch on one sampler (eight chunks per
-    row, the finisher hand-off), the inputs changed before the first, the
-    wrapping and the last calls, each of those checked against the
-    oracle."""
+    row, the finisher hand-off; at top-k 50 the waves' speculative keys too),
+    the inputs changed before the first, the wrapping and the last calls,
+    each of those checked against the oracle."""
     import torch
     monkeypatch.setenv("FG_HIP_TARGET_GROUPS", "16")
     rows, vocab = 2, 8192
     s = fg_hip.HipSampler(vocab, rows)
-    s.set_configs([fg_hip.make_config(0.9, 0.9, 16, 0.0, 0.0, 1.0)] * rows)
+    s.set_configs([fg_hip.make_config(0.9, 0.9, top_k, 0.0, 0.0, 1.0)] * rows)
     tok = torch.empty(rows, dtype=torch.int32, device=dev)
     st = torch.empty(rows, dtype=torch.int32, device=dev)
     checks = {0, 8189, 8190, 8191, 8192, 8199}
@@ -661,7 +662,7 @@ def test_finisher_epoch_wrap(dev, monkeypatch):
             rng = np.random.default_rng(call)
             w = dict(logits=rng.normal(0, 2, (rows, vocab)).astype(np.float32),
                      counts=np.zeros((rows, vocab), dtype=np.uint32),
-                     configs=[W.cfg(0.9, 0.9, 16)] * rows,
+                     configs=[W.cfg(0.9, 0.9, top_k)] * rows,
                      uniforms=rng.random(rows).astype(np.float32), logprobs=0)
             x, u = to_dev(w["logits"], dev), to_dev(w["uniforms"], dev)
         s.sample(x, u, tok, row_status=st)
