@@ -14,15 +14,22 @@
 //             moves (the reference's per-tile select, shaders/fg_topk_select.comp,
 //             recast as a streaming merge);
 //   * log-probs: per-lane online (max, sum exp) in f32.
-// Row hand-off: when a row spans several workgroups, every wave publishes its
-// top-kk list, greedy winner and (max, sum) with device-coherent (sc1) stores
-// and waits for them; the workgroup then bumps the row's arrival counter (one
-// cache line per row, so rows never contend).  The last workgroup to arrive
-// reads the row's partials with sc1 loads, merges the sorted lists and runs
-// the select arithmetic of src/sampler.c:80-122 in one wave, then resets the
-// row's counter for the next launch.  No L2 write-back or invalidate is
-// needed.  A row that fits one workgroup is
-// merged straight from LDS.
+// Row hand-off, when a row spans several workgroups (one workgroup's row is
+// merged straight from LDS):
+//   * the finisher: batches whose rows all keep top lists of at most 64 over
+//     2-8 chunks, or are all greedy over 2-64, in a launch that fits the device
+//     at once and is not being captured.  Every chunk but one leaves its list
+//     as words tagged with the launch's epoch and ends; that one reads until
+//     every word carries the tag, within a limit.
+//   * the last arriver: every other batch.  A workgroup publishes its top-kk
+//     list, greedy winner and (max, sum) with device-coherent (sc1) stores,
+//     waits for them and bumps the row's arrival counter (one cache line per
+//     row, so rows never contend).  The last to arrive reads the row's partials
+//     with sc1 loads, and resets the counter for the next launch.  No L2
+//     write-back or invalidate is needed, and nobody waits.
+// Lists of up to 8 chunks are merged, those of more are selected from
+// (many_select; log-prob and whole-row nucleus launches merge them too); the
+// select arithmetic of src/sampler.c:80-122 then runs in one wave.
 #pragma once
 
 #include "fg_device.hpp"

@@ -171,10 +171,10 @@ void fg_sampler_hip_destroy(fg_sampler_hip *sampler);
  * that hand-off one workgroup of each row waits, on the device, for the
  * row's other workgroups (it is used only when the whole launch fits on the
  * device at once, for batches of greedy rows and for batches of top-k rows
- * over at most 8 workgroups each; any other batch waits for nobody); a row whose wait passes the limit gets row_status
- * FG_ERR_UNAVAILABLE and token 0xffffffff instead of a token.  0 makes
- * every such row that is not complete at the first look report it (a
- * host-side way to exercise that path). */
+ * over at most 8 workgroups each; any other batch waits for nobody).  A row
+ * whose wait passes the limit gets row_status FG_ERR_UNAVAILABLE and token
+ * 0xffffffff instead of a token.  0 makes every such row that is not complete
+ * at the first look report it (a host-side way to exercise that path). */
 fg_status fg_sampler_hip_set_wait_limit(fg_sampler_hip *sampler, uint64_t wait_us, fg_error *err);
 
 /* Validates each row's controls as fg_sampler_config_validate does and keeps
@@ -387,8 +387,9 @@ fg_status fg_hip_output_slice_run_dense(fg_hip_output_slice *slice, const void *
  * controls").  Two launches per pass of up to 64 tokens (the product, then
  * the sampler over its logits, which stay in the slice's workspace: 64 MB at
  * most, allocated at create; wider vocabularies take fewer tokens a pass, and
- * so does a slice created when memory is short).  Nothing in it waits for another workgroup, so
- * row_status is never FG_ERR_UNAVAILABLE.  Calls on one slice must not
+ * so does a slice created when memory is short).  Nothing in it waits for
+ * another workgroup, so row_status is never FG_ERR_UNAVAILABLE and no wait
+ * limit applies.  Calls on one slice must not
  * overlap.  The history increment stays a separate step
  * (fg_sampler_hip_history_increment, or the caller's own). */
 fg_status fg_hip_output_slice_run_dense_sampled(
