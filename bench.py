@@ -1,6 +1,6 @@
 """Benchmark of the batched sampler on one MI355X.
 
-Default workload: BASELINE.json config 2 (the north star) -- 64 rows x
+Default workload: benchmark configuration 2 -- 64 rows x
 151,936 f32 logits N(0, 3^2) with 5 ids/row boosted by +8, per-row history
 counts from 1,024 Zipf(1.1) ids, presence 1.5 + repetition 1.05, T 0.7,
 top-k 20, top-p 0.8, one uniform per row.  A step is one fg_sampler_hip_sample
@@ -21,10 +21,9 @@ head (248,320 x 2,560 Q8_0 weights in the cooked layout, random bytes with
 binary16 scales in [1e-3, 2e-2]) times `--tokens` hidden vectors, fused with
 each token's greedy finalist (fg_hip_output_slice_run_dense, ways 1).
 
-`--config N` times the other configurations of BASELINE.json the same way
+`--config N` times the other configurations the same way
 (1: one greedy row; 3: 256 rows, whole-row nucleus; 4: 128 rows, quantised
-logits, greedy or sampled; 5: 1,024 rows with top-20 log-probs).  The driver
-runs the default.
+logits, greedy or sampled; 5: 1,024 rows with top-20 log-probs).
 
 Output: one JSON line (see the repository's bench contract), with `roofline`
 (dominant kernel: algorithmic bytes / HIP-event launch time vs the 8 TB/s HBM
@@ -75,7 +74,7 @@ def zipf_counts(torch, g, dev, rows, draws, perm, vocab=VOCAB):
 
 
 class Workload:
-    """One BASELINE.json configuration: row count, per-row controls, input
+    """One benchmark configuration: row count, per-row controls, input
     generator and the algorithmic bytes of one step."""
 
     def __init__(self, cid, fg_hip, sampled=True):
@@ -506,7 +505,7 @@ def main():
     ap.add_argument("--gpus", type=int, default=1)
     ap.add_argument("--steps", type=int, default=2000)
     ap.add_argument("--warmup", type=int, default=100)
-    ap.add_argument("--config", type=int, default=2, help="BASELINE.json configuration (1-5)")
+    ap.add_argument("--config", type=int, default=2, help="benchmark configuration (1-5)")
     ap.add_argument("--greedy", action="store_true", help="config 4: the greedy run")
     ap.add_argument("--set-gb", type=float, default=4.0, help="distinct input bytes to rotate over")
     ap.add_argument("--cpu-seconds", type=float, default=12.0)

@@ -1,4 +1,4 @@
-"""bench.py end to end at the driver's short settings: the run must emit one
+"""bench.py end to end at short settings: the run must emit one
 parsed JSON line whose batch-0 parity check and row-status check passed,
 whatever the number of steps (a short run writes only some rotated sets)."""
 import json

@@ -2,7 +2,7 @@
 per case (greedy, top-k 1-64, whole-row nucleus and log-probs mixed or alone;
 penalties on some rows; ties, plateaus and non-finite values; vocabularies
 that split unevenly; 1-64 workgroups per row and both row hand-offs), each
-against the C oracle on the same inputs at the north-star bar (ids exact
+against the C oracle on the same inputs at the same bar as the fixed cases (ids exact
 except within 1e-6 of a boundary; 1e-11 for whole-row nucleus rows, whose
 masses are summed differently).  The cases are fixed by their seeds."""
 import numpy as np

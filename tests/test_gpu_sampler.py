@@ -1,7 +1,7 @@
 """GPU parity: the HIP batched sampler (C ABI fg_sampler_hip_sample) against the
 CPU oracle on identical inputs and identical per-row uniforms.
 
-Bar (BASELINE.json north_star): token ids bit-exact, except where the oracle's
+Bar: token ids bit-exact, except where the oracle's
 f64 running sums come within 1e-6 (relative) of a top-p or draw boundary;
 penalised logits within 1e-6 relative (the C rounding is reproduced exactly, so
 the check is bit-exact); log-probs within 1e-5 absolute.
@@ -18,7 +18,7 @@ BOUNDARY = 1e-6
 LP_TOL = 1e-5
 # Whole-row nucleus masses are summed with an f64 exp of a few ulp: tokens
 # must match the oracle except where its sums come within 1e-11 of a
-# boundary (1e-6, would excuse most deep cuts, whose
+# boundary (the bar, 1e-6, would excuse most deep cuts, whose
 # steps are ~1e-5 of the mass each).
 NUC_BOUNDARY = 1e-11
 

@@ -1,4 +1,4 @@
-"""Synthetic inputs of the five BASELINE.json configs, built with the oracle's
+"""Synthetic inputs of the five benchmark configurations, built with the oracle's
 Philox4x32-10 generators so CPU and GPU see identical bytes.  `rows` and `vocab`
 can be reduced for oracle-speed parity tests; seeds are 1001..1005."""
 from __future__ import annotations
